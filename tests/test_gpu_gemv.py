@@ -44,6 +44,22 @@ def test_dequant_bit_exact(qh, oracle, t):
     assert np.array_equal(got.view(np.uint32), ref.view(np.uint32))
 
 
+@pytest.mark.parametrize("t", ALL_TYPES)
+@pytest.mark.parametrize("blocks", [1, 3, 129, 1025])
+def test_dequant_bit_exact_ragged(qh, oracle, t, blocks):
+    """Partial workgroups and steps, a tail of n % 4 for the one-element types, an
+    output at a 4-byte boundary and blocks at an odd byte address."""
+    _, qk, bb = GGML_TYPES[t]
+    n = blocks * qk
+    data = synth.weights(t, blocks, qk, seed=200 + t)
+    w = GpuBuf.upload(np.concatenate([np.zeros(1, np.uint8), data]))
+    out = GpuBuf.upload_f32(np.full(n + 2, 7.0))
+    check("hip_dequant", qh.hip_dequant(t, w.ptr + 1, out.ptr + 4, n))
+    got = out.download(np.float32)
+    assert got[0] == 7.0 and got[n + 1] == 7.0
+    assert np.array_equal(got[1:n + 1].view(np.uint32), oracle.dequant(t, data, n).view(np.uint32))
+
+
 def test_dequant_f16_all_patterns(qh, oracle):
     bits = np.arange(65536, dtype=np.uint16).view(np.uint8)
     w = GpuBuf.upload(bits)
