@@ -14,7 +14,7 @@ pytestmark = pytest.mark.gpu
 
 @pytest.mark.parametrize("t", [12, 14])
 @pytest.mark.parametrize("rows, in_dim, out_dim", [(1, 256, 37), (3, 1024, 300), (16, 4096, 64), (17, 512, 129),
-                                                   (40, 2048, 16)])
+                                                   (40, 2048, 16), (33, 768, 257), (130, 256, 128)])
 @pytest.mark.parametrize("stream_k", [None, (128, 2), (300, 7)])
 def test_gemm_q8_1_mmq_bit_exact(qh, oracle, t, rows, in_dim, out_dim, stream_k):
     rng = np.random.default_rng(rows * 7 + in_dim + out_dim + t)
