@@ -165,8 +165,8 @@ hipError_t qh_launch_gemv(uint32_t type, const uint8_t* W, const float* x, float
     return hipGetLastError();
 }
 
-// Batched tokens: the matrix-core kernel (one weight pass per 16 tokens) where
-// it covers the type and shape, else one batch-1 pass per token.
+// Batched tokens: the superblock formats' matrix-core kernel (one weight pass per
+// 32 tokens), the block formats' (16 tokens), else one batch-1 pass per token.
 hipError_t qh_launch_gemm(uint32_t type, const uint8_t* W, const float* x, float* y, int in_dim, int out_dim,
                           int n, hipStream_t st) {
     if (n == 1) return qh_launch_gemv(type, W, x, y, in_dim, out_dim, st);
@@ -174,6 +174,8 @@ hipError_t qh_launch_gemm(uint32_t type, const uint8_t* W, const float* x, float
     if (type == QT_F32) return qh_launch_gemm_f32(reinterpret_cast<const float*>(W), x, y, in_dim, out_dim, n, st);
     if (!qh_force_valu()) {
         hipError_t e = qh_launch_mmq(type, W, x, y, in_dim, out_dim, n, st);
+        if (e != hipErrorNotSupported) return e;
+        e = qh_launch_mmb(type, W, x, y, in_dim, out_dim, n, st);
         if (e != hipErrorNotSupported) return e;
     }
     for (int t = 0; t < n; t++) {

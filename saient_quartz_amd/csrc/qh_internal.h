@@ -48,6 +48,8 @@ hipError_t qh_launch_mmv16(uint32_t type, const uint8_t* W, const float* x, floa
                            hipStream_t st);
 hipError_t qh_launch_mmq(uint32_t type, const uint8_t* W, const float* x, float* y, int in_dim, int out_dim,
                          int n, hipStream_t st);
+hipError_t qh_launch_mmb(uint32_t type, const uint8_t* W, const float* x, float* y, int in_dim, int out_dim, int n,
+                         hipStream_t st);
 hipError_t qh_launch_mmq_mixed(uint32_t t1, int c1, const uint8_t* const* W1, float* const* Y1, const int* o1,
                                uint32_t t2, int c2, const uint8_t* const* W2, float* const* Y2, const int* o2,
                                const float* x, int n, int in_dim, hipStream_t st, const float* nw = nullptr);
