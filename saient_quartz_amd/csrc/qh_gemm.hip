@@ -86,8 +86,9 @@ QH_DEV qh_f16x8 qg_cvt8(uint32_t w0, uint32_t w1, qh_f16x2 scv, qh_f16x2 cv) {
 // ---------------------------------------------------------------- formats
 // Each format gives BYTES, CH (16-byte slices staged per row and superblock,
 // the last from byte LAST), RS (LDS line per row), the header decoded once per
-// group (hdr: d, dmin, scales) and bop<J>: lane half hh's B operand of K-block
-// J (weights 16 J + 8 hh .. + 7 of the lane's row) from the staged line r.
+// group (hdr: d, dmin, scales) and lane half hh's B operand of K-block J (weights
+// 16 J + 8 hh .. + 7 of the lane's row) in two steps: raw<J>, the bytes from the
+// staged line r, and cvt<J>.
 
 // Q4_K (src/dequant.rs:1471-1519): sub-block sb = 2p + nibble uses qs[32p + l].
 struct GQ4K {
@@ -106,10 +107,14 @@ struct GQ4K {
         o.dm = qh_f16_hi(h.x);
         return o;
     }
+    using Raw = qh_u32x2;
     template <int J>
-    static QH_DEV qh_f16x8 bop(const unsigned char* r, int hh, const H& h, const unsigned char*) {
-        constexpr int sb = J >> 1, jj = J & 1, p = sb >> 1, nib = sb & 1;
-        const qh_u32x2 w = *reinterpret_cast<const qh_u32x2*>(r + 16 + 32 * p + 16 * jj + 8 * hh);
+    static QH_DEV Raw raw(const unsigned char* r, int hh) {
+        return *reinterpret_cast<const qh_u32x2*>(r + 16 + 32 * (J >> 2) + 16 * (J & 1) + 8 * hh);
+    }
+    template <int J>
+    static QH_DEV qh_f16x8 cvt(const Raw& w, const H& h, const unsigned char*) {
+        constexpr int sb = J >> 1, nib = sb & 1;
         const uint32_t q0 = nib ? (w.x >> 4) & 0x0F0F0F0Fu : w.x & 0x0F0F0F0Fu;
         const uint32_t q1 = nib ? (w.y >> 4) & 0x0F0F0F0Fu : w.y & 0x0F0F0F0Fu;
         const qh_f16x2 scv = qg_dup(sb < 4 ? h.sc0 : h.sc1, sb & 3, (_Float16)1024.0f);
@@ -123,6 +128,13 @@ struct GQ4K {
         const qh_f16x2 c = qg_dup(m, 2, (_Float16)1024.0f), d = qg_dup(m, 3, (_Float16)1024.0f);
         return qh_f16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
     }
+    // the 8 mins, one per K position (both lane halves alike)
+    static QH_DEV qh_f16x8 minw(const H& h) {
+        const qh_f16x2 k = {(_Float16)1024.0f, (_Float16)1024.0f};
+        const qh_f16x2 a = qg_b2h(h.mn0, QG_SEL01) - k, b = qg_b2h(h.mn0, QG_SEL23) - k;
+        const qh_f16x2 c = qg_b2h(h.mn1, QG_SEL01) - k, d = qg_b2h(h.mn1, QG_SEL23) - k;
+        return qh_f16x8{a[0], a[1], b[0], b[1], c[0], c[1], d[0], d[1]};
+    }
 };
 
 // Q5_K (src/dequant.rs:1146-1182): as Q4_K plus bit sb of qh[l] as bit 4.
@@ -132,17 +144,23 @@ struct GQ5K {
     static constexpr int GRID = 0;
     using H = GQ4K::H;
     static QH_DEV H hdr(const unsigned char* r) { return GQ4K::hdr(r); }
+    struct Raw { qh_u32x2 w, u; };
     template <int J>
-    static QH_DEV qh_f16x8 bop(const unsigned char* r, int hh, const H& h, const unsigned char*) {
-        constexpr int sb = J >> 1, jj = J & 1, p = sb >> 1, nib = sb & 1;
-        const qh_u32x2 w = *reinterpret_cast<const qh_u32x2*>(r + 48 + 32 * p + 16 * jj + 8 * hh);
-        const qh_u32x2 u = *reinterpret_cast<const qh_u32x2*>(r + 16 + 16 * jj + 8 * hh);
+    static QH_DEV Raw raw(const unsigned char* r, int hh) {
+        return Raw{*reinterpret_cast<const qh_u32x2*>(r + 48 + 32 * (J >> 2) + 16 * (J & 1) + 8 * hh),
+                   *reinterpret_cast<const qh_u32x2*>(r + 16 + 16 * (J & 1) + 8 * hh)};
+    }
+    template <int J>
+    static QH_DEV qh_f16x8 cvt(const Raw& v, const H& h, const unsigned char*) {
+        constexpr int sb = J >> 1, nib = sb & 1;
+        const qh_u32x2 w = v.w, u = v.u;
         const uint32_t q0 = (nib ? (w.x >> 4) & 0x0F0F0F0Fu : w.x & 0x0F0F0F0Fu) | (((u.x >> sb) & 0x01010101u) << 4);
         const uint32_t q1 = (nib ? (w.y >> 4) & 0x0F0F0F0Fu : w.y & 0x0F0F0F0Fu) | (((u.y >> sb) & 0x01010101u) << 4);
         const qh_f16x2 scv = qg_dup(sb < 4 ? h.sc0 : h.sc1, sb & 3, (_Float16)1024.0f);
         return qg_cvt8(q0, q1, scv, scv * (_Float16)-1024.0f);
     }
     static QH_DEV qh_f16x8 minh(const H& h, int hh) { return GQ4K::minh(h, hh); }
+    static QH_DEV qh_f16x8 minw(const H& h) { return GQ4K::minw(h); }
 };
 
 // Q6_K (src/dequant.rs:1583-1631): weight 128 h + 32 k + l (h < 2, k < 4, l <
@@ -162,13 +180,18 @@ struct GQ6K {
         o.dm = 0.f;
         return o;
     }
+    struct Raw { qh_u32x2 ql, qh; };
     template <int J>
-    static QH_DEV qh_f16x8 bop(const unsigned char* r, int hh, const H& h, const unsigned char*) {
+    static QH_DEV Raw raw(const unsigned char* r, int hh) {
         constexpr int hf = J >> 3, k = (J >> 1) & 3, l0 = 16 * (J & 1);
-        const qh_u32x2 ql = *reinterpret_cast<const qh_u32x2*>(r + 64 * hf + 32 * (k & 1) + l0 + 8 * hh);
-        const qh_u32x2 qh = *reinterpret_cast<const qh_u32x2*>(r + 128 + 32 * hf + l0 + 8 * hh);
-        const uint32_t q0 = ((ql.x >> (4 * (k >> 1))) & 0x0F0F0F0Fu) | (((qh.x >> (2 * k)) & 0x03030303u) << 4);
-        const uint32_t q1 = ((ql.y >> (4 * (k >> 1))) & 0x0F0F0F0Fu) | (((qh.y >> (2 * k)) & 0x03030303u) << 4);
+        return Raw{*reinterpret_cast<const qh_u32x2*>(r + 64 * hf + 32 * (k & 1) + l0 + 8 * hh),
+                   *reinterpret_cast<const qh_u32x2*>(r + 128 + 32 * hf + l0 + 8 * hh)};
+    }
+    template <int J>
+    static QH_DEV qh_f16x8 cvt(const Raw& v, const H& h, const unsigned char*) {
+        constexpr int k = (J >> 1) & 3;
+        const uint32_t q0 = ((v.ql.x >> (4 * (k >> 1))) & 0x0F0F0F0Fu) | (((v.qh.x >> (2 * k)) & 0x03030303u) << 4);
+        const uint32_t q1 = ((v.ql.y >> (4 * (k >> 1))) & 0x0F0F0F0Fu) | (((v.qh.y >> (2 * k)) & 0x03030303u) << 4);
         // the signed scale as an f16 pair: byte ^ 0x80 is sc + 128
         const qh_f16x2 scv = qg_dup(h.s[J >> 2] ^ 0x80808080u, J & 3, (_Float16)1152.0f);
         const qh_f16x2 m32 = {(_Float16)-1056.0f, (_Float16)-1056.0f};
@@ -196,16 +219,19 @@ struct GIQ3S {
     static constexpr int GRID = 1;
     struct H { float d, dm; };
     static QH_DEV H hdr(const unsigned char* r) { return H{qh_h2f(qh_rd16(r, 0)), 0.f}; }
+    struct Raw { uint32_t q, qh, sg, sc; };  // 2 grid indices, their 9th bits, 8 sign bits, the scales byte
     template <int J>
-    static QH_DEV qh_f16x8 bop(const unsigned char* r, int hh, const H&, const unsigned char* tab) {
+    static QH_DEV Raw raw(const unsigned char* r, int hh) {
         constexpr int K = J >> 1, jj = J & 1;
-        const uint32_t q = qh_rd16(r, 2 + 8 * K + 4 * jj + 2 * hh);                   // 2 grid indices
-        const uint32_t qh = (uint32_t)r[66 + K] >> (4 * jj + 2 * hh);                  // their 9th bits
-        const uint32_t sg = (uint32_t)r[qh_iq3s_at(74 + 4 * K + 2 * jj + hh)];         // 8 sign bits
-        const qh_u32x2 g0 = *reinterpret_cast<const qh_u32x2*>(tab + 8 * ((q & 0xFFu) | ((qh & 1u) << 8)));
-        const qh_u32x2 g1 = *reinterpret_cast<const qh_u32x2*>(tab + 8 * (((q >> 8) & 0xFFu) | ((qh & 2u) << 7)));
-        const qh_u32x4 m = *reinterpret_cast<const qh_u32x4*>(tab + IQT_SIGN + 16 * sg);
-        const int sc = 1 + 2 * (int)((r[qh_iq3s_at(106 + K / 2)] >> (4 * (K & 1))) & 0xFu);
+        return Raw{qh_rd16(r, 2 + 8 * K + 4 * jj + 2 * hh), (uint32_t)r[66 + K] >> (4 * jj + 2 * hh),
+                   r[qh_iq3s_at(74 + 4 * K + 2 * jj + hh)], r[qh_iq3s_at(106 + K / 2)]};
+    }
+    template <int J>
+    static QH_DEV qh_f16x8 cvt(const Raw& v, const H&, const unsigned char* tab) {
+        const qh_u32x2 g0 = *reinterpret_cast<const qh_u32x2*>(tab + 8 * ((v.q & 0xFFu) | ((v.qh & 1u) << 8)));
+        const qh_u32x2 g1 = *reinterpret_cast<const qh_u32x2*>(tab + 8 * (((v.q >> 8) & 0xFFu) | ((v.qh & 2u) << 7)));
+        const qh_u32x4 m = *reinterpret_cast<const qh_u32x4*>(tab + IQT_SIGN + 16 * v.sg);
+        const int sc = 1 + 2 * (int)((v.sc >> (4 * ((J >> 1) & 1))) & 0xFu);
         const qh_f16x2 scv = {(_Float16)sc, (_Float16)sc};
         const qh_f16x2 a = qg_u2h(g0.x ^ m.x) * scv, b = qg_u2h(g0.y ^ m.y) * scv;
         const qh_f16x2 c = qg_u2h(g1.x ^ m.z) * scv, d = qg_u2h(g1.y ^ m.w) * scv;
@@ -219,15 +245,18 @@ struct GIQ2XXS {
     static constexpr int GRID = 2;
     struct H { float d, dm; };
     static QH_DEV H hdr(const unsigned char* r) { return H{0.125f * qh_h2f(qh_rd16(r, 0)), 0.f}; }
+    struct Raw { uint32_t idx, a1, s7; };  // grid index, the sub-block's sign and scale word, this group's signs
     template <int J>
-    static QH_DEV qh_f16x8 bop(const unsigned char* r, int hh, const H&, const unsigned char* tab) {
+    static QH_DEV Raw raw(const unsigned char* r, int hh) {
         constexpr int K = J >> 1, jj = J & 1;
-        const uint32_t idx = r[2 + 8 * K + 2 * jj + hh];
         const uint32_t a1 = qh_rd16(r, qh_iq2xxs_at(6 + 8 * K)) | (qh_rd16(r, qh_iq2xxs_at(8 + 8 * K)) << 16);
-        const qh_u32x4 g = *reinterpret_cast<const qh_u32x4*>(tab + 16 * idx);
-        const uint32_t s8 = qh_ksigns((a1 >> (7 * (2 * jj + hh))) & 127u);
-        const qh_u32x4 m = *reinterpret_cast<const qh_u32x4*>(tab + IQT_SIGN + 16 * s8);
-        const int sc = 2 * (int)(a1 >> 28) + 1;
+        return Raw{r[2 + 8 * K + 2 * jj + hh], a1, (a1 >> (7 * (2 * jj + hh))) & 127u};
+    }
+    template <int J>
+    static QH_DEV qh_f16x8 cvt(const Raw& v, const H&, const unsigned char* tab) {
+        const qh_u32x4 g = *reinterpret_cast<const qh_u32x4*>(tab + 16 * v.idx);
+        const qh_u32x4 m = *reinterpret_cast<const qh_u32x4*>(tab + IQT_SIGN + 16 * qh_ksigns(v.s7));
+        const int sc = 2 * (int)(v.a1 >> 28) + 1;
         const qh_f16x2 scv = {(_Float16)sc, (_Float16)sc};
         const qh_f16x2 a = qg_u2h(g.x ^ m.x) * scv, b = qg_u2h(g.y ^ m.y) * scv;
         const qh_f16x2 c = qg_u2h(g.z ^ m.z) * scv, d = qg_u2h(g.w ^ m.w) * scv;
@@ -383,11 +412,26 @@ static __device__ __align__(256) unsigned int qh_mmq_cnt[QG_PART_TILES * QG_WAVE
 //     which makes the token's results NaN).
 // Tokens past the block's n write nothing (their rows are never read back
 // into results).
-// Digitise one 8-element chunk of the image: token t = xt, elements 8 xc ..
-// 8 xc + 7 of the group (xc < 32), values v; the 32 lanes of a token form one
-// half of a wavefront and must all take part (lanes with `on` false hold
-// zeros and write nothing).  `im` is the group's image (global or LDS).
-QH_DEV void qg_digitise(const float* v, bool on, int lane, int xt, int xc, unsigned char* im) {
+// One 8-element chunk (xc = 0 .. 31 of a group) of one token, split into f16: the
+// chunk's hi and lo pairs, the sub-block's x sum (hi and lo, low halves of p5 and
+// q5; sub-block xc / 4) and the token's exponent s; `bad` when the token's group
+// holds an Inf or NaN.  The 32 lanes of a token form one half of a wavefront and
+// must all take part (lanes without a token hold zeros).  RN: hi and lo rounded to
+// nearest, where an extra instruction per element does not count: x then keeps 23
+// bits instead of the 22 of two truncations.
+struct QgSplit {
+    uint32_t hi[4], lo[4];
+    uint32_t sum;  // the sum's hi f16 and, in the upper half, its lo
+    int s;
+    bool bad;
+};
+template <bool RN>
+QH_DEV qh_f16x2 qg_f16x2(float a, float b) {
+    if constexpr (RN) return qh_f16x2{(_Float16)a, (_Float16)b};
+    return __builtin_bit_cast(qh_f16x2, __builtin_amdgcn_cvt_pkrtz(a, b));
+}
+template <bool RN>
+QH_DEV QgSplit qg_split(const float* v, int lane) {
     float m = 0.f, sum = 0.f;
     bool fin = true;
 #pragma unroll
@@ -403,39 +447,46 @@ QH_DEV void qg_digitise(const float* v, bool on, int lane, int xt, int xc, unsig
     m = fmaxf(m, __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(m), 0x140, 0xF, 0xF, false)));
     m = fmaxf(m, __shfl_xor(m, 16));
     const uint64_t bad = __ballot(!fin);
-    const bool fb = ((bad >> (lane & 32)) & 0xFFFFFFFFull) != 0;
+    QgSplit o;
+    o.bad = ((bad >> (lane & 32)) & 0xFFFFFFFFull) != 0;
     int e = 0;
     (void)frexpf(m, &e);
     int s = m > 0.f ? 14 - e : 0;
     s = s > 126 ? 126 : (s < -126 ? -126 : s);
+    o.s = s;
     const float scx = ldexpf(1.0f, s);
-    uint32_t hi4[4], lo4[4];
 #pragma unroll
     for (int i = 0; i < 4; i++) {
         const float a = v[2 * i] * scx, b = v[2 * i + 1] * scx;
-        const auto hp = __builtin_amdgcn_cvt_pkrtz(a, b);
-        const auto lp = __builtin_amdgcn_cvt_pkrtz(a - (float)hp[0], b - (float)hp[1]);
-        hi4[i] = __builtin_bit_cast(uint32_t, hp);
-        lo4[i] = __builtin_bit_cast(uint32_t, lp);
+        const qh_f16x2 hp = qg_f16x2<RN>(a, b);
+        const qh_f16x2 lp = qg_f16x2<RN>(a - (float)hp[0], b - (float)hp[1]);
+        o.hi[i] = __builtin_bit_cast(uint32_t, hp);
+        o.lo[i] = __builtin_bit_cast(uint32_t, lp);
     }
-    const int u = xc >> 1, c = xc & 1;
     // sub-block sb = xc / 4: the sum over 4 lanes (a DPP quad)
     sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0xB1, 0xF, 0xF, false));
     sum += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(sum), 0x4E, 0xF, 0xF, false));
     const float s5 = sum * ldexpf(1.0f, s - 5);
-    const auto p5 = __builtin_amdgcn_cvt_pkrtz(s5, 0.f);
-    const auto q5 = __builtin_amdgcn_cvt_pkrtz(s5 - (float)p5[0], 0.f);
+    const qh_f16x2 p5 = qg_f16x2<RN>(s5, 0.f), q5 = qg_f16x2<RN>(s5 - (float)p5[0], 0.f);
+    o.sum = (uint32_t)__builtin_bit_cast(uint16_t, p5[0]) | ((uint32_t)__builtin_bit_cast(uint16_t, q5[0]) << 16);
+    return o;
+}
+// Digitise one 8-element chunk of the image: token t = xt, elements 8 xc ..
+// 8 xc + 7 of the group (xc < 32), values v; the 32 lanes of a token form one
+// half of a wavefront and must all take part (lanes with `on` false hold
+// zeros and write nothing).  `im` is the group's image (global or LDS).
+QH_DEV void qg_digitise(const float* v, bool on, int lane, int xt, int xc, unsigned char* im) {
+    const QgSplit x = qg_split<false>(v, lane);
+    const int u = xc >> 1, c = xc & 1;
     if (!on) return;
-    *reinterpret_cast<qh_u32x4*>(im + 1024 * u + 16 * (2 * xt + 32 * c)) = qh_u32x4{hi4[0], hi4[1], hi4[2], hi4[3]};
-    *reinterpret_cast<qh_u32x4*>(im + 1024 * u + 16 * (2 * xt + 1 + 32 * c)) = qh_u32x4{lo4[0], lo4[1], lo4[2], lo4[3]};
+    *reinterpret_cast<qh_u32x4*>(im + 1024 * u + 16 * (2 * xt + 32 * c)) = qh_u32x4{x.hi[0], x.hi[1], x.hi[2], x.hi[3]};
+    *reinterpret_cast<qh_u32x4*>(im + 1024 * u + 16 * (2 * xt + 1 + 32 * c)) = qh_u32x4{x.lo[0], x.lo[1], x.lo[2], x.lo[3]};
     const int sb = xc >> 2;
-    if ((xc & 3) == 0) {
-        const uint32_t pair = (uint32_t)__builtin_bit_cast(uint16_t, p5[0]) | ((uint32_t)__builtin_bit_cast(uint16_t, q5[0]) << 16);
-        *reinterpret_cast<uint32_t*>(im + XImg::SUM + 16 * (xt + 16 * (sb >> 2)) + 4 * (sb & 3)) = pair;
-    }
+    if ((xc & 3) == 0)
+        *reinterpret_cast<uint32_t*>(im + XImg::SUM + 16 * (xt + 16 * (sb >> 2)) + 4 * (sb & 3)) = x.sum;
     if (xc == 0)
         reinterpret_cast<float*>(im + XImg::RSF)[8 * ((xt >> 1) & 1) + 2 * (xt >> 2) + (xt & 1)] =
-            fb ? __builtin_nanf("") : ldexpf(1.0f, -s);
+            x.bad ? __builtin_nanf("") : ldexpf(1.0f, -x.s);
 }
 
 // x (and the SwiGLU up operand x2) of one token chunk: 8 floats at p (and p2).
@@ -708,7 +759,7 @@ __device__ __forceinline__ void qh_mmq_body(const QgGroups& gs, const QgXs& xs, 
         }
         auto kb = [&](auto JC) {
             constexpr int J = decltype(JC)::value;
-            const qh_f16x8 b = F::template bop<J>(wrow, hh, hd, gridl);
+            const qh_f16x8 b = F::template cvt<J>(F::template raw<J>(wrow, hh), hd, gridl);
 #pragma unroll
             for (int h = 0; h < NTH; h++) {
                 const qh_f16x8 a = __builtin_bit_cast(qh_f16x8, qh_lds128(im + h * XI::BYTES + 1024 * J + 16 * lane));
@@ -1119,11 +1170,21 @@ static hipError_t qg_run(uint32_t type, const QgEntry* en, int cnt, int in_dim, 
     return hipGetLastError();
 }
 
+// Prompts (qh_mmw.hip).  QwImgs: whose images the image array holds, within one
+// call (x null: nobody's).
+struct QwImgs {
+    const float *x, *x2;
+    int n;
+};
+hipError_t qw_run(uint32_t type, const uint8_t* W, const float* X, const float* X2, float* Y, int n, int rows, int in_dim,
+                  int accum, const QgScratch& sc, QwImgs* have, hipStream_t st);
+
 // Batched tokens on the matrix cores for `count` matrices of one type and
 // in_dim: Y[i][t][:] = W[i] X[i][t][:] for t < n[i] (token-major, y token stride
 // out_dims[i]); hipErrorNotSupported when the type/shape has no kernel here.
-// Tokens go in chunks of up to 16 (one weight pass each); matrices whose
-// weights pass 2 GB go in row chunks.  The split-K partials and counters are
+// Matrices with enough tokens go through the wide kernel (qw_run), the others in
+// chunks of up to 32 tokens (one weight pass each); matrices whose weights pass
+// 2 GB go in row chunks.  The split-K partials and counters are
 // one array per device, so calls that overlap on one device (different
 // streams) must be serialised by the caller.
 hipError_t qh_launch_mmq_grouped(uint32_t type, int count, const uint8_t* const* W, const float* const* X,
@@ -1163,8 +1224,15 @@ hipError_t qh_launch_mmq_grouped(uint32_t type, int count, const uint8_t* const*
     QgEntry batch[QG_MAXG];
     int cnt = 0, slots = 0;
     const float* last_x = nullptr;
+    QwImgs have = {nullptr, nullptr, 0};
     for (int i = 0; i < count; i++) {
         if (out_dims[i] <= 0) continue;
+        if (n[i] > 32) {
+            hipError_t e = qw_run(type, W[i], X[i], X2 ? X2[i] : nullptr, Y[i], n[i], out_dims[i], in_dim, accum, *sc, &have, st);
+            if (e == hipSuccess) continue;
+            if (e != hipErrorNotSupported) return e;
+        }
+        have.x = nullptr;
         for (int t0 = 0; t0 < n[i]; t0 += 32) {
             // blocks of up to 32 tokens (17-32: one weight pass on two halves)
             const int nt = n[i] - t0 < 32 ? n[i] - t0 : 32;
