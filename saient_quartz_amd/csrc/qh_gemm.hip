@@ -39,6 +39,7 @@
 #include "qh_internal.h"
 
 typedef float qh_f32x16 __attribute__((ext_vector_type(16)));
+typedef float qh_f32x4 __attribute__((ext_vector_type(4)));
 typedef _Float16 qh_f16x8 __attribute__((ext_vector_type(8)));
 typedef _Float16 qh_f16x2 __attribute__((ext_vector_type(2)));
 
@@ -1063,6 +1064,27 @@ static int qg_pick_splits(int blocks, int ngroups, int gmax, int target) {
     return best;
 }
 
+// Up to 16 tokens and few rows (qh_mms.hip): matrices that share one x, whose images
+// are in slot 0.  qs_pick: whether it is faster than qh_mmq.
+#define QS_MAXM 8
+struct QsMat {
+    uint32_t type;
+    const uint8_t* w;
+    float* y;
+    int rows, ldy;
+};
+bool qs_pick(const QsMat* ms, int cnt, int in_dim, int n);
+hipError_t qs_run(const QsMat* ms, int cnt, const unsigned char* img, int n, int in_dim, int accum, hipStream_t st);
+// The images of one block of n <= 16 tokens into slot 0.
+static void qg_image16(const float* x, const float* x2, int n, int in_dim, const QgScratch& sc, hipStream_t st) {
+    QgXs xs = {};
+    xs.halves = 1;
+    xs.x[0] = x;
+    xs.x2[0] = x2;
+    xs.n[0] = n;
+    hipLaunchKernelGGL(qg_ximage, dim3((unsigned)(in_dim / 256), 1), dim3(512), 0, st, xs, sc.img, in_dim);
+}
+
 // One grouped launch: every entry's row blocks, each workgroup digitising its
 // own K split of its entry's x.
 // img_ready: the launch's one token block already has its images in slot 0
@@ -1093,6 +1115,14 @@ static hipError_t qg_run(uint32_t type, const QgEntry* en, int cnt, int in_dim, 
         gs.x2[i] = en[i].x2;
         gs.n[i] = en[i].n;
         ntmax = en[i].n > ntmax ? en[i].n : ntmax;
+    }
+    if (nslots == 1 && ntmax <= 16 && cnt <= QS_MAXM && qh_mmq_mode_env() < 0 && qh_mmq_splits_env() <= 0) {
+        QsMat ms[QS_MAXM];
+        for (int i = 0; i < cnt; i++) ms[i] = QsMat{type, en[i].w, en[i].y, en[i].rows, en[i].ldy};
+        if (qs_pick(ms, cnt, in_dim, ntmax)) {
+            if (!img_ready) qg_image16(en[0].x, en[0].x2, ntmax, in_dim, sc, st);
+            return qs_run(ms, cnt, sc.img, ntmax, in_dim, accum, st);
+        }
     }
     // One 32-row tile per wavefront, QG_WAVES per workgroup.  Splits: enough
     // workgroups for one per CU (the kernel's registers allow no second).
@@ -1338,6 +1368,20 @@ hipError_t qh_launch_mmq_mixed(uint32_t t1, int c1, const uint8_t* const* W1, fl
     for (int i = 0; i < c2; i++) {
         if (o2[i] <= 0 || (int64_t)o2[i] * rb2 >= ((int64_t)1 << 31) - 4096) return hipErrorNotSupported;
         b2 += (o2[i] + brows - 1) / brows;
+    }
+    if (n <= 16 && c1 + c2 <= QS_MAXM && qh_mmq_mode_env() < 0 && qh_mmq_splits_env() <= 0) {
+        QsMat ms[QS_MAXM];
+        for (int i = 0; i < c1; i++) ms[i] = QsMat{t1, W1[i], Y1[i], o1[i], o1[i]};
+        for (int i = 0; i < c2; i++) ms[c1 + i] = QsMat{t2, W2[i], Y2[i], o2[i], o2[i]};
+        if (qs_pick(ms, c1 + c2, in_dim, n)) {
+            if (nw) {
+                hipError_t e = qh_glue_norm_image(sc->img, x, nw, n, in_dim, st);
+                if (e != hipSuccess) return e;
+            } else {
+                qg_image16(x, nullptr, n, in_dim, *sc, st);
+            }
+            return qs_run(ms, c1 + c2, sc->img, n, in_dim, 0, st);
+        }
     }
     const int smin = (ngroups + QG_GMAX - 1) / QG_GMAX;
     int s1 = 0, s2 = 0;

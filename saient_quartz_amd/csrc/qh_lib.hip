@@ -7,6 +7,7 @@
 #include "qh_mmv16.hip"
 #include "qh_gemm.hip"
 #include "qh_mmw.hip"
+#include "qh_mms.hip"
 #include "qh_mmb.hip"
 #include "qh_mmq81.hip"
 #include "qh_gemv.hip"

@@ -2,7 +2,7 @@
 sizes) on Q4_K, Q5_K, Q6_K, IQ3_S and IQ2_XXS, against float64 sums of the
 closed-form weights on a sample of rows (both ends, tile edges, the middle).
 
-Bound: x is kept to 21 bits per element (relative 2^-21, truncated), so an
+Bound: x is kept to at least 21 bits per element (relative 2^-21), so an
 output's error is at most 2^-21 sum |w x| plus f32 rounding of the sums; the
 2-norm over the sampled outputs is held to 2^-20 of that sum's norm, with a
 format's scaled quant and its minimum counted apart.
