@@ -36,6 +36,10 @@ typedef int32_t qh_i32x4 __attribute__((ext_vector_type(4)));
 #define QH_XG 1024
 #define QH_XG_SUM 768
 #define QH_XG_ZERO 832
+// Formats with DIG4 keep x as four digits (31 bits below the largest |x|): plane 3 takes
+// the sums' place (they have no minimums) and the zero bytes follow it.
+#define QH_XG4 1040
+#define QH_XG4_ZERO 1024
 #define QH_RS 240   // LDS line per row: 15 x 16 bytes, conflict-free b128 reads over 16 rows
 #define QH_MAXT 64  // row tiles per workgroup (their results wait in LDS until the end)
 #define QH_RING 4   // finished tiles per workgroup barrier (launches with few tiles)
@@ -52,6 +56,12 @@ template <class F, class = void>
 struct QhHalf : std::false_type {};
 template <class F>
 struct QhHalf<F, std::void_t<decltype(F::HALF)>> : std::bool_constant<F::HALF> {};
+template <class F, class = void>
+struct QhDig4 : std::false_type {};
+template <class F>
+struct QhDig4<F, std::void_t<decltype(F::DIG4)>> : std::bool_constant<F::DIG4> {};
+template <class F>
+constexpr int qh_xg() { return QhDig4<F>::value ? QH_XG4 : QH_XG; }
 QH_DEV uint32_t qh_hi4(uint32_t q) { return (q >> 4) & 0x0F0F0F0Fu; }
 
 // ---------------------------------------------------------------- formats
@@ -308,16 +318,17 @@ struct M16IQ2XXS {
 // p / 2, 16 quants as the int8 B operand with the block's own f32 scale d
 // (FLOAT_D); the offset of Q4_0 / Q5_0 (-8 / -16) and IQ4_NL's codebook go into
 // the bytes, the minimum m of Q4_1 / Q5_1 through the piece's x sum.
-// Dispatched for Q4_1 and Q5_1 only: their quants sit 4- and 8-byte aligned in
-// the staged line; the 18- and 22-byte blocks of Q4_0, IQ4_NL and Q5_0 leave
-// them 2-byte aligned, and those measured no faster (Q5_0: 23.4 against 15.1 us
-// at 14336x4096) than the VALU kernel, which keeps them.
+// The quants of Q4_1 and Q5_1 sit 4- and 8-byte aligned in the staged line; the 18-
+// and 22-byte blocks of Q4_0, IQ4_NL and Q5_0 put every second block's 2 bytes past a
+// dword: whole dwords are read and shifted (read as they lie, Q5_0 14336 x 4096 took
+// 23.4 us).  These three, which the VALU kernel computes in f32 otherwise, take four
+// digits of x, in the A rows that a fourth digit finds free.
 template <int KIND>  // 0 Q4_0, 1 Q4_1, 2 Q5_0, 3 Q5_1, 4 IQ4_NL
 struct M16Blk {
     static constexpr int BB = (KIND == 0 || KIND == 4) ? 18 : (KIND == 1 ? 20 : (KIND == 2 ? 22 : 24));
     static constexpr int QS = (KIND == 0 || KIND == 4) ? 2 : (KIND == 1 ? 4 : (KIND == 2 ? 6 : 8));  // quants
     static constexpr int BYTES = 8 * BB, CH = BYTES / 16, ROWS = 128 / CH, LAST = BYTES - 16, RS = QH_RS;
-    static constexpr bool FLOAT_D = true, MINS = KIND == 1 || KIND == 3;
+    static constexpr bool FLOAT_D = true, MINS = KIND == 1 || KIND == 3, DIG4 = !MINS;
     static constexpr int GRID = 0;
     struct H { float d[4], m[4]; float dm; };
     template <int S>
@@ -337,14 +348,18 @@ struct M16Blk {
 #pragma unroll
         for (int s = 0; s < 4; s++) {
             const int p = 4 * s + kg, blk = p >> 1, half = p & 1;
-            uint32_t w[4];
-            __builtin_memcpy(w, r + BB * blk + QS, 16);
-            uint32_t hb = 0;
-            if constexpr (KIND == 2 || KIND == 3) {
-                uint32_t qh;
-                __builtin_memcpy(&qh, r + BB * blk + QS - 4, 4);
-                hb = half ? qh >> 16 : qh & 0xFFFFu;  // bit j: weight j of the piece
+            uint32_t w[4], qh = 0;
+            if constexpr (BB % 4 == 0) {
+                __builtin_memcpy(w, r + BB * blk + QS, 16);
+                if constexpr (KIND == 3) __builtin_memcpy(&qh, r + BB * blk + QS - 4, 4);
+            } else {  // even blocks' quants lie 2 bytes past a dword
+                const uint32_t sh = (blk & 1) ? 0u : 2u;
+                const uint32_t* a = reinterpret_cast<const uint32_t*>(r + BB * blk + QS - sh);
+#pragma unroll
+                for (int i = 0; i < 4; i++) w[i] = __builtin_amdgcn_alignbyte(a[i + 1], a[i], sh);
+                if constexpr (KIND == 2) qh = __builtin_amdgcn_alignbyte(a[0], a[-1], sh);
             }
+            const uint32_t hb = half ? qh >> 16 : qh & 0xFFFFu;  // bit j: weight j of the piece
 #pragma unroll
             for (int i = 0; i < 4; i++) {
                 uint32_t q = half ? (w[i] >> 4) & 0x0F0F0F0Fu : w[i] & 0x0F0F0F0Fu;
@@ -372,6 +387,8 @@ struct M16Blk {
 struct M16Q4K16 : M16Q4K { static constexpr int ROWS = 16; };
 struct M16Q5K16 : M16Q5K { static constexpr int ROWS = 16; };
 struct M16Q8016 : M16Q80 { static constexpr int ROWS = 16; };
+template <int KIND>
+struct M16Blk16 : M16Blk<KIND> { static constexpr int ROWS = 16; };
 
 // ---------------------------------------------------------------- kernel
 
@@ -440,7 +457,7 @@ constexpr int qh_maxt() { return NT > 2 ? 8 : (NT > 1 ? 16 : QH_MAXT); }
 // ring of wavefront partials, finished rows and the per-wavefront sums of x^2.
 template <class F, int W, int GPW, int NT = 1>
 constexpr int qh_mmv16_lds() {
-    return W * GPW * (F::ROWS * F::RS + 16) + W * GPW * NT * QH_XG + 2 * qh_ring<NT>() * W * 16 * 4 * NT +
+    return W * GPW * (F::ROWS * F::RS + 16) + W * GPW * NT * qh_xg<F>() + 2 * qh_ring<NT>() * W * 16 * 4 * NT +
            qh_maxt<NT>() * 16 * 4 * NT + W * 4 * NT + (F::GRID ? 2048 : 0);
 }
 
@@ -451,6 +468,9 @@ __device__ __forceinline__ void qh_mmv16_body(const QhMats& mm, const QhOne& one
                                               uint32_t row_bytes, int ngroups, unsigned char* lds, const int bid,
                                               const int nblk) {
     static_assert(!PAIR || NT == 1, "SwiGLU pairs run one token");
+    constexpr bool DIG4 = QhDig4<F>::value;
+    static_assert(!DIG4 || (F::FLOAT_D && !F::MINS), "four digits: float scales, no sums");
+    constexpr int XG = qh_xg<F>(), XG_ZERO = DIG4 ? QH_XG4_ZERO : QH_XG_ZERO;
     constexpr int RING = qh_ring<NT>();
     constexpr int ROWS = F::ROWS, CH = F::CH;
     constexpr int NH = (ROWS * CH + 63) / 64;  // 16-byte loads per lane and group
@@ -463,9 +483,9 @@ __device__ __forceinline__ void qh_mmv16_body(const QhMats& mm, const QhOne& one
     const int ntok = NT == 1 ? 1 : mm.ntok;
     const QhBuf xb = qh_buf(x, 4u * (256u * (uint32_t)ngroups + (NT > 1 ? (uint32_t)(mm.ldx * (ntok - 1)) : 0u)));
     unsigned char* wl = lds + w * (GPW * TILE);  // GPW staging tiles of this wavefront
-    // x digit planes of group t, token k at xl + (t NT + k) QH_XG
-    unsigned char* xl = lds + W * GPW * TILE + w * (GPW * NT * QH_XG);
-    float* red = reinterpret_cast<float*>(lds + W * GPW * TILE + W * GPW * NT * QH_XG);
+    // x digit planes of group t, token k at xl + (t NT + k) XG
+    unsigned char* xl = lds + W * GPW * TILE + w * (GPW * NT * XG);
+    float* red = reinterpret_cast<float*>(lds + W * GPW * TILE + W * GPW * NT * XG);
     float* res = red + 2 * RING * W * 16 * NT;  // finished rows of this workgroup's tiles
     float* sqw = res + qh_maxt<NT>() * 16 * NT;  // per-wavefront sums of x^2 (fused RMS norm)
     unsigned char* gridl = reinterpret_cast<unsigned char*>(sqw + W * NT);  // IQ codebook (GRID formats)
@@ -514,11 +534,11 @@ __device__ __forceinline__ void qh_mmv16_body(const QhMats& mm, const QhOne& one
     // (set after the first loads are issued: see set_offsets)
     uint32_t aoff[4], xsoff[4];
     auto set_offsets = [&]() {
-        const bool arow = (n >> 2) == kg && (n & 3) < 3;
-        aoff[0] = arow ? 256u * (n & 3) + 16u * F::template piece<0>(kg) : QH_XG_ZERO;
-        aoff[1] = arow ? 256u * (n & 3) + 16u * F::template piece<1>(kg) : QH_XG_ZERO;
-        aoff[2] = arow ? 256u * (n & 3) + 16u * F::template piece<2>(kg) : QH_XG_ZERO;
-        aoff[3] = arow ? 256u * (n & 3) + 16u * F::template piece<3>(kg) : QH_XG_ZERO;
+        const bool arow = (n >> 2) == kg && (DIG4 || (n & 3) < 3);
+        aoff[0] = arow ? 256u * (n & 3) + 16u * F::template piece<0>(kg) : XG_ZERO;
+        aoff[1] = arow ? 256u * (n & 3) + 16u * F::template piece<1>(kg) : XG_ZERO;
+        aoff[2] = arow ? 256u * (n & 3) + 16u * F::template piece<2>(kg) : XG_ZERO;
+        aoff[3] = arow ? 256u * (n & 3) + 16u * F::template piece<3>(kg) : XG_ZERO;
         xsoff[0] = QH_XG_SUM + 4u * F::template piece<0>(kg);
         xsoff[1] = QH_XG_SUM + 4u * F::template piece<1>(kg);
         xsoff[2] = QH_XG_SUM + 4u * F::template piece<2>(kg);
@@ -631,32 +651,38 @@ __device__ __forceinline__ void qh_mmv16_body(const QhMats& mm, const QhOne& one
         m = qh_dpp_max(m);
         int e = 0;
         (void)frexpf(m, &e);
-        int s = m > 0.f ? 22 - e : 0;
+        int s = m > 0.f ? (DIG4 ? 30 : 22) - e : 0;
         s = s > 126 ? 126 : s;
         const float scx = ldexpf(1.0f, s);
         const uint32_t bias = 0x4B400000u - 0x808080u;
 #pragma unroll
         for (int t = 0; t < GPW; t++) {
             const float4 v = xall[t * NT + k];
-            unsigned char* xp = xl + (t * NT + k) * QH_XG;
-            const uint32_t a0 = (__float_as_uint(fmaf(v.x, scx, 12582912.0f)) - bias) ^ 0x808080u;
-            const uint32_t a1 = (__float_as_uint(fmaf(v.y, scx, 12582912.0f)) - bias) ^ 0x808080u;
-            const uint32_t a2 = (__float_as_uint(fmaf(v.z, scx, 12582912.0f)) - bias) ^ 0x808080u;
-            const uint32_t a3 = (__float_as_uint(fmaf(v.w, scx, 12582912.0f)) - bias) ^ 0x808080u;
+            unsigned char* xp = xl + (t * NT + k) * XG;
+            auto digits = [&](float f) -> uint32_t {
+                if constexpr (DIG4) return ((uint32_t)__float2int_rn(f * scx) + 0x808080u) ^ 0x808080u;
+                else return (__float_as_uint(fmaf(f, scx, 12582912.0f)) - bias) ^ 0x808080u;
+            };
+            const uint32_t a0 = digits(v.x), a1 = digits(v.y), a2 = digits(v.z), a3 = digits(v.w);
             const uint32_t t01 = __builtin_amdgcn_perm(a1, a0, 0x05010400u);
             const uint32_t t23 = __builtin_amdgcn_perm(a3, a2, 0x05010400u);
-            const uint32_t u01 = __builtin_amdgcn_perm(a1, a0, 0x06020602u);
-            const uint32_t u23 = __builtin_amdgcn_perm(a3, a2, 0x06020602u);
+            constexpr uint32_t UP = DIG4 ? 0x07030602u : 0x06020602u;
+            const uint32_t u01 = __builtin_amdgcn_perm(a1, a0, UP);
+            const uint32_t u23 = __builtin_amdgcn_perm(a3, a2, UP);
             // lane holds x[256t + 4 lane .. +3] = positions 4(lane%4).. of piece lane/4.
             unsigned char* ub = xp + 4 * lane;
             *reinterpret_cast<uint32_t*>(ub) = __builtin_amdgcn_perm(t23, t01, 0x05040100u);
             *reinterpret_cast<uint32_t*>(ub + 256) = __builtin_amdgcn_perm(t23, t01, 0x07060302u);
             *reinterpret_cast<uint32_t*>(ub + 512) = __builtin_amdgcn_perm(u23, u01, 0x05040100u);
-            float hs = (v.x + v.y) + (v.z + v.w);
-            hs += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(hs), 0xB1, 0xF, 0xF, false));
-            hs += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(hs), 0x4E, 0xF, 0xF, false));
-            if ((lane & 3) == 0) *reinterpret_cast<float*>(xp + QH_XG_SUM + lane) = hs;
-            if (lane == 0) *reinterpret_cast<qh_u32x4*>(xp + QH_XG_ZERO) = qh_u32x4{0, 0, 0, 0};
+            if constexpr (DIG4) {
+                *reinterpret_cast<uint32_t*>(ub + 768) = __builtin_amdgcn_perm(u23, u01, 0x07060302u);
+            } else {
+                float hs = (v.x + v.y) + (v.z + v.w);
+                hs += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(hs), 0xB1, 0xF, 0xF, false));
+                hs += __int_as_float(__builtin_amdgcn_update_dpp(0, __float_as_int(hs), 0x4E, 0xF, 0xF, false));
+                if ((lane & 3) == 0) *reinterpret_cast<float*>(xp + QH_XG_SUM + lane) = hs;
+            }
+            if (lane == 0) *reinterpret_cast<qh_u32x4*>(xp + XG_ZERO) = qh_u32x4{0, 0, 0, 0};
         }
         return ldexpf(1.0f, -s);
     };
@@ -709,14 +735,15 @@ __device__ __forceinline__ void qh_mmv16_body(const QhMats& mm, const QhOne& one
             for (int k = 0; k < NT; k++) {
                 int i0 = 0, i1 = 0, i2 = 0;
                 float fm = 0.f;
-                const unsigned char* xt = xl + (t * NT + k) * QH_XG;
+                const unsigned char* xt = xl + (t * NT + k) * XG;
                 auto mfma = [&](auto SC) {
                     constexpr int S = decltype(SC)::value;
                     const qh_i32x4 a = *reinterpret_cast<const qh_i32x4*>(xt + aoff[S]);
                     const qh_i32x4 D = __builtin_amdgcn_mfma_i32_16x16x64_i8(a, B[S], qh_i32x4{0, 0, 0, 0}, 0, 0, 0);
                     if constexpr (F::FLOAT_D) {
                         // each piece has its own f32 scale (the digit dots are exact in f32)
-                        const float P = fmaf((float)D[2], 65536.0f, fmaf((float)D[1], 256.0f, (float)D[0]));
+                        const float P = DIG4 ? fmaf((float)(D[3] * 256 + D[2]), 65536.0f, (float)(D[1] * 256 + D[0]))
+                                             : fmaf((float)D[2], 65536.0f, fmaf((float)D[1], 256.0f, (float)D[0]));
                         acc[k] = fmaf(F::template dsc<S>(hd), P, acc[k]);
                         if constexpr (F::MINS) {
                             const float xs = *reinterpret_cast<const float*>(xt + xsoff[S]);
@@ -1090,6 +1117,22 @@ static bool qh_rows16_better(int rows, int out_dim) {
     return ((rb + cus - 1) / cus) * 16 < ((ra + cus - 1) / cus) * rows;
 }
 
+// Q4_0, Q5_0, IQ4_NL with a K that gives every wavefront a group and enough weights for
+// the chip (us, VALU kernel / here: Q5_0 4096 x 14336 17.6 / 11.5, 14336 x 4096 14.2 /
+// 10.6, 2000 x 8448 14.2 / 8.7, 4096 x 4096 5.65 / 5.59; Q4_0 4096 x 14336 16.7 / 10.3;
+// IQ4_NL 17.9 / 12.1).  Others stay with the VALU kernel (Q5_0 1024 x 4096 4.7 / 4.9,
+// 8192 x 2048 6.2 / 7.0, 50000 x 2304 28 / 36).  Bound by the integer products' operands
+// from LDS (two byte shifts a dword); error against 64 bits, Q5_0 4096 x 14336: VALU
+// 2.1e-7, here 9.9e-8 (three digits of x: 8e-7).
+template <int KIND>
+static hipError_t blk_mmv16(const uint8_t* W, const float* x, float* y, int in_dim, int out_dim, uint32_t row_bytes,
+                            hipStream_t st) {
+    if (in_dim < 4096 || (int64_t)in_dim * out_dim < (1 << 24)) return hipErrorNotSupported;
+    return qh_rows16_better(M16Blk<KIND>::ROWS, out_dim)
+               ? dispatch_mmv16<M16Blk16<KIND>>(W, x, y, in_dim, out_dim, row_bytes, st)
+               : dispatch_mmv16<M16Blk<KIND>>(W, x, y, in_dim, out_dim, row_bytes, st);
+}
+
 // Returns hipErrorNotSupported when the type/shape has no kernel here.
 hipError_t qh_launch_mmv16(uint32_t type, const uint8_t* W, const float* x, float* y, int in_dim, int out_dim,
                            hipStream_t st) {
@@ -1108,6 +1151,9 @@ hipError_t qh_launch_mmv16(uint32_t type, const uint8_t* W, const float* x, floa
             return in_dim <= 4096 ? dispatch_mmv16<M16Q6K>(W, x, y, in_dim, out_dim, row_bytes, st)
                                   : dispatch_mmv16<M16Q6KW>(W, x, y, in_dim, out_dim, row_bytes, st);
         case QT_IQ3_S: return dispatch_mmv16<M16IQ3S>(W, x, y, in_dim, out_dim, row_bytes, st);
+        case QT_Q4_0: return blk_mmv16<0>(W, x, y, in_dim, out_dim, row_bytes, st);
+        case QT_Q5_0: return blk_mmv16<2>(W, x, y, in_dim, out_dim, row_bytes, st);
+        case QT_IQ4_NL: return blk_mmv16<4>(W, x, y, in_dim, out_dim, row_bytes, st);
         case QT_Q4_1: return dispatch_mmv16<M16Blk<1>>(W, x, y, in_dim, out_dim, row_bytes, st);
         case QT_Q5_1: return dispatch_mmv16<M16Blk<3>>(W, x, y, in_dim, out_dim, row_bytes, st);
         case QT_IQ2_XXS: return dispatch_mmv16<M16IQ2XXS>(W, x, y, in_dim, out_dim, row_bytes, st);
