@@ -87,8 +87,8 @@ int hip_gemv_fused_async(uint32_t ggml_type, int count, const uint8_t* const* W,
 
 /* Y[t][j] = sum_k W[j,k] X[t][k] for t < n (token-major).  GPU counterpart of
  * dequant::gemm (src/dequant.rs:143-200); n == 1 is hip_gemv.  For n >= 2 the
- * matrix-core path reads the weights once per 32 tokens (see the note above on
- * its device scratch); x is kept to 23 bits below each token's largest |x| per
+ * matrix-core paths read the weights once per 16 tokens (32-element blocks), per 32
+ * or, for prompts, once per launch (see the note above on the device scratch); x is kept to 23 bits below each token's largest |x| per
  * 256 elements, so results stay within 1e-3 relative L2 per token (observed
  * ~1e-6) with activation outliers up to thousands of times the RMS. */
 int hip_gemm(uint32_t ggml_type, const uint8_t* d_data, const float* d_x, float* d_y, int in_dim, int out_dim,
